@@ -14,7 +14,7 @@ __global__ __launch_bounds__(TI* TJ) void k_lxw_flux(LxwArgs a, int ntj)
     if (lxw_halted(a)) return;
     const int ti = blockIdx.x / ntj, tj = blockIdx.x - ti * ntj;
     const int e0i = ti * TI, e0j = tj * TJ;
-    lxw_phase_load<P, TI, TJ, R>(threadIdx.x, e0i, e0j, a, sm);
+    lxw_phase_load<P, TI, TJ, R>(threadIdx.x, TI * TJ, e0i, e0j, a, sm);
     __syncthreads();
     lxw_phase_cell<P, TI, TJ, R>(threadIdx.x, e0i, e0j, a, sm);
 }

@@ -247,6 +247,18 @@ __host__ __device__ __forceinline__ void lxw_phase_load(int tid, int e0i, int e0
     }
 }
 
+// The same for a workgroup of nthreads threads (at most TI TJ, whose shares of
+// the cells they take in turn).
+template <class P, int TI, int TJ, typename R = double>
+__host__ __device__ __forceinline__ void lxw_phase_load(int tid, int nthreads, int e0i, int e0j, const LxwArgs& a,
+                                                        LxwSmem<TI, TJ, P::MEQN, R>& sm)
+{
+    do {
+        lxw_phase_load<P, TI, TJ, R>(tid, e0i, e0j, a, sm);
+        tid += nthreads;
+    } while (tid < TI * TJ);
+}
+
 template <typename R>
 __host__ __device__ __forceinline__ R d1(R h, R f0, R f1, R f3, R f4)
 {

@@ -253,6 +253,36 @@ int emu_construct_integrated_r(const finess_params* p, double dt, const double* 
     return 0;
 }
 
+// ConstructIntegratedR through the LxW kernel's phases with `nthreads` threads
+// loading a tile.
+int emu_integrated_threads(const finess_params* p, double dt, const double* q, int nthreads, double* F, double* G)
+{
+    const int M = 5, g = p->mbc;
+    std::vector<double> qg = to_planes_ghosted(p, q, M);
+    const long long le = p->my + 6, lpl = (long long)(p->mx + 6) * le, ldq = p->my + 2 * g;
+    std::vector<double> Fo((size_t)M * lpl), Go((size_t)M * lpl);
+    LxwArgs a;
+    memset(&a, 0, sizeof a);
+    a.q = qg.data(); a.src_ghosts = g; a.F = Fo.data(); a.G = Go.data(); a.mx = p->mx; a.my = p->my;
+    a.plane = (long long)p->mx * p->my; a.time_order = p->time_order; a.dt = dt; a.dx = p->dx; a.dy = p->dy;
+    a.pp.gamma = p->gamma;
+    const int nti = (p->mx + 6 + LTI - 1) / LTI, ntj = (p->my + 6 + LTJ - 1) / LTJ;
+    std::vector<LxwSmem<LTI, LTJ, 5>> smv(1);
+    for (int t = 0; t < nti * ntj; t++) {
+        const int e0i = (t / ntj) * LTI, e0j = (t % ntj) * LTJ;
+        for (int tid = 0; tid < nthreads; tid++) lxw_phase_load<Euler2D, LTI, LTJ>(tid, nthreads, e0i, e0j, a, smv[0]);
+        for (int tid = 0; tid < LTI * LTJ; tid++) lxw_phase_cell<Euler2D, LTI, LTJ>(tid, e0i, e0j, a, smv[0]);
+    }
+    for (int i = -3; i < p->mx + 3; i++)
+        for (int j = -3; j < p->my + 3; j++)
+            for (int m = 0; m < M; m++) {
+                const long long o = (long long)m * lpl + (long long)(i + 3) * le + (j + 3);
+                F[((i + g) * ldq + (j + g)) * M + m] = Fo[o];
+                G[((i + g) * ldq + (j + g)) * M + m] = Go[o];
+            }
+    return 0;
+}
+
 // ConstructIntegratedR through the FP64 form's phases (lxw64_*).
 int emu_integrated_fp64(const finess_params* p, double dt, const double* q, double* F, double* G)
 {
