@@ -138,9 +138,14 @@ extern "C" int finess_construct_l_planes_noalloc(const finess_params* pin, const
                    : p.weno_version == FINESS_WENO_Z ? weno_z5_kind(p.power_param, p.epsilon)
                    : p.power_param == 2.0 ? WENO_JS5_P2 : WENO_JS5_POW;
     const int rc = launch_stage2d(p.physics, p.precision == FINESS_PREC_FP32, wk, 0, a, st);
-    if (rc) return rc == -1 ? FINESS_ERR_CONFIG : FINESS_ERR_HIP;
-    hipLaunchKernelGGL(k_fold_cfl_words, dim3(1), dim3(64), 0, st, cfl, smax2);
-    if (hipGetLastError() == hipSuccess) return FINESS_OK;
-    launch_fill_u64(cfl, 2 * CFL_SPREAD, 0ull, st);  // the stage's maxima must not reach the next call
+    if (rc == -1) return FINESS_ERR_CONFIG;  // nothing launched
+    if (!rc) {
+        hipLaunchKernelGGL(k_fold_cfl_words, dim3(1), dim3(64), 0, st, cfl, smax2);
+        if (hipGetLastError() == hipSuccess) return FINESS_OK;
+    }
+    // A launch that reports an error may have run all the same (the error can be
+    // an earlier one that the thread had not read): the stage's maxima must not
+    // reach the next call.
+    launch_fill_u64(cfl, 2 * CFL_SPREAD, 0ull, st);
     return FINESS_ERR_HIP;
 }
