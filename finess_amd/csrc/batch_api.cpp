@@ -95,8 +95,12 @@ int set_shape(finess_batch* b, int shape)
         map.insert(map.end(), (size_t)nti * pr.ntj, k);
     }
     if ((int)map.size() > b->tile_cap) {
+        // the graph's kernels hold the old map's address
+        if (b->exec) hipGraphExecDestroy(b->exec);
+        b->exec = nullptr;
         hipFree(b->tile_prob);
         b->tile_prob = nullptr;
+        b->tile_cap = 0;
         if (hipMalloc((void**)&b->tile_prob, map.size() * sizeof(int)) != hipSuccess)
             return bfail(b, FINESS_ERR_HIP, "tile map allocation failed");
         b->tile_cap = (int)map.size();
