@@ -116,12 +116,15 @@ struct finess_ctx {
     double last_ms = 0.0;
     long long last_launches = 0;
     std::string err;
-    // large state downloads (download_large): pinned slots and their events
+    // large state downloads (download): pinned slots and their events
+    static constexpr int PIN_SLOTS = 8;
     char* pin = nullptr;
-    std::vector<hipEvent_t> pin_ev;
+    hipEvent_t pin_ev[PIN_SLOTS] = {};
 };
 
 namespace {
+
+constexpr int PIN_SLOTS = finess_ctx::PIN_SLOTS;
 
 constexpr int NSLOT = 8;
 
@@ -794,28 +797,37 @@ int ensure_ghosted(finess_ctx* c)
 
 // Downloads of at least DOWNLOAD_LARGE bytes: the device copies run ahead
 // into pinned slots while several threads move finished slots to the caller's
-// memory.  That memory is as a rule fresh, and a single thread that faults its
-// pages in while it copies reaches 10 GB/s of the link's 57: the state of a
-// 2048^2 Euler grid (169 MB) took 17 ms that way.
-constexpr size_t DOWNLOAD_LARGE = (size_t)8 << 20, PIN_SLOT = (size_t)2 << 20;
-constexpr int PIN_SLOTS = 8, COPY_THREADS = 8;
+// memory.  Memory of that size is as a rule fresh (glibc maps every block
+// beyond 32 MiB anew), and a single thread that faults its pages in while it
+// copies reaches 10 GB/s of the link's 57.  Milliseconds per read, plain copy
+// and slots: 169 MB 16.8 / 4.8, 42 MB 4.3 / 1.5, 33 MB 2.6 / 1.6, 21 MB
+// 1.6 / 1.0.  A context's first read also makes the slots, which takes 1.0 to
+// 1.5 ms: 42 MB 4.4 / 3.0, but 33 MB 2.8 / 3.3 and 21 MB 1.9 / 2.8 (into memory
+// that is not fresh 34 MB 2.6 / 2.1).  The line lies where that first read is
+// the faster one too.
+constexpr size_t DOWNLOAD_LARGE = (size_t)32 << 20, PIN_SLOT = (size_t)2 << 20;
+constexpr int COPY_THREADS = 8;
 
-// Prepares the pinned slots; false (and nothing changed) if they cannot be had.
+// Prepares the pinned slots; false (and no error left on the thread) if they
+// cannot be had.  The events belong to the context's device, whatever device
+// the calling thread has current.
 bool ensure_pinned(finess_ctx* c)
 {
     if (c->pin) return true;
-    while (c->pin_ev.size() < (size_t)PIN_SLOTS) {
-        hipEvent_t e;
-        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) return false;
-        c->pin_ev.push_back(e);
-    }
-    void* p = nullptr;
-    if (hipHostMalloc(&p, PIN_SLOT * PIN_SLOTS, hipHostMallocDefault) != hipSuccess) {
+    int dev = 0;
+    bool ok = hipGetDevice(&dev) == hipSuccess && (dev == c->device || hipSetDevice(c->device) == hipSuccess);
+    if (!ok) {
         (void)hipGetLastError();
         return false;
     }
-    c->pin = static_cast<char*>(p);
-    return true;
+    for (int k = 0; k < PIN_SLOTS && ok; k++)
+        ok = c->pin_ev[k] || hipEventCreateWithFlags(&c->pin_ev[k], hipEventDisableTiming) == hipSuccess;
+    void* p = nullptr;
+    ok = ok && hipHostMalloc(&p, PIN_SLOT * PIN_SLOTS, hipHostMallocDefault) == hipSuccess;
+    if (!ok) (void)hipGetLastError();
+    if (dev != c->device && hipSetDevice(dev) != hipSuccess) (void)hipGetLastError();
+    c->pin = ok ? static_cast<char*>(p) : nullptr;
+    return ok;
 }
 
 // dst (host) = src (device), n bytes, after the work enqueued on c->st.
@@ -1304,7 +1316,8 @@ void finess_destroy(finess_ctx* c)
     hipFree(c->route_flux);
     if (c->smax_h) hipHostFree(c->smax_h);
     if (c->pin) hipHostFree(c->pin);
-    for (hipEvent_t e : c->pin_ev) hipEventDestroy(e);
+    for (hipEvent_t e : c->pin_ev)
+        if (e) hipEventDestroy(e);
     for (hipEvent_t e : c->tev) hipEventDestroy(e);
     if (c->ev0) hipEventDestroy(c->ev0);
     if (c->ev1) hipEventDestroy(c->ev1);
