@@ -266,10 +266,20 @@ __global__ __launch_bounds__(SMALL1D_NT) void k_run1d_small(Stage1DRun r)
 // 200 cells take 2.1 us per step; the kernel above took 6.9 (two barriers, flux
 // and state through generic pointers and the boundary map per stencil cell,
 // the controller behind a third barrier): a chain of latencies, on one CU.
-// 400 cells 3.1 (8.6), 1000 6.8 (13.3), 2000 10.0 and 2700 12.5 (31 with
+// 400 cells 3.1 (8.6), 1000 5.8 (13.3), 2000 9.6 and 2700 11.7 (32 with
 // two launches per stage), which RUN1D_CELLS takes as far as the 64 KB of LDS
 // that a launch gets without an attribute.
-constexpr int RUN1D_CELLS = 2700, RUN1D_WAVES = 16, RUN1D_CHUNK = 31;
+//
+// More than 16 x 31 cells take all 16 waves, whose last chunks may hold no
+// cells and are then left out: four waves on each SIMD share the chunks evenly
+// (1000 cells in nine waves of four chunks: 7.4 us; 520 cells 3.9, now 3.4).
+//
+// The kinds with pow, which are bound by its instructions on the one CU, stop
+// at RUN1D_CELLS_POW, the limit of the step kernels: 1000 cells take 34.7 us
+// (41.7 in the kernel above), 1536 48.6 (65.6).  Beyond, two launches per stage
+// take 31 to 38; the run took 60 at 1600 cells and 89 at 2700 (before the even
+// sharing of the chunks, which gave a fifth at most).
+constexpr int RUN1D_CELLS = 2700, RUN1D_CELLS_POW = 1536, RUN1D_WAVES = 16, RUN1D_CHUNK = 31;
 
 // lane i takes lane i + 1's value (the last keeps its own)
 __device__ __forceinline__ double wave_next(double v)
@@ -316,6 +326,10 @@ __global__ __launch_bounds__(RUN1D_WAVES * 64) void k_run1d_wave(Stage1DRun r)
     const Stage1DArgs& a = r.base;
     const int n = a.mx, ld = n + 6, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
     const int part = lane & 1;
+    // the wave's chunks that hold cells; the first FULL always do (launch_run1d)
+    constexpr int FULL = NCH <= 2 ? NCH - 1 : NCH - 2;
+    const int first = RUN1D_CHUNK * __builtin_amdgcn_readfirstlane(wave);
+    const int chunks = first < n ? (n - first + nw * RUN1D_CHUNK - 1) / (nw * RUN1D_CHUNK) : 0;
     double* const X = run1d_lds;             // the two copies, ld apart
     double* const haux = run1d_lds + 2 * ld; // half the advection speeds
     for (int i = (int)threadIdx.x - 3; i < n + 3; i += blockDim.x) {
@@ -354,6 +368,7 @@ __global__ __launch_bounds__(RUN1D_WAVES * 64) void k_run1d_wave(Stage1DRun r)
             double* const D = X + s * ld;
 #pragma unroll
             for (int c = 0; c < NCH; c++) {
+                if (NCH > 1 && c >= FULL && c >= chunks) continue;
                 // part 0: cells f-3..f+1, part 1: f+2..f-2
                 const int i0 = part ? face[c] + 5 : face[c], st = part ? -1 : 1;
                 double v[5];
@@ -395,7 +410,7 @@ __global__ __launch_bounds__(RUN1D_WAVES * 64) void k_run1d_wave(Stage1DRun r)
 template <int WK, int NCH>
 static void launch_run1d_wave(const Stage1DRun& r, hipStream_t st)
 {
-    const int nw = (r.base.mx + NCH * RUN1D_CHUNK - 1) / (NCH * RUN1D_CHUNK);
+    const int nw = NCH > 1 ? RUN1D_WAVES : (r.base.mx + RUN1D_CHUNK - 1) / RUN1D_CHUNK;
     hipLaunchKernelGGL((k_run1d_wave<WK, NCH>), dim3(1), dim3(nw * 64), 3 * (r.base.mx + 6) * sizeof(double), st, r);
 }
 
@@ -496,6 +511,7 @@ int launch_run1d(int wk, const Stage1DRun& r, hipStream_t st)
 
 bool run1d_fits(int wk, int mx)
 {
+    if (wk == WENO_JS5_POW || wk == WENO_Z5) return mx <= RUN1D_CELLS_POW;
     if (wk < WENO_JS7) return mx <= RUN1D_CELLS;
     // (and the run's LDS within the 64 KB a launch gets without an attribute)
     return run1d_lds_bytes(mx) + 2048 <= 65536 &&
