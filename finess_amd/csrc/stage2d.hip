@@ -52,7 +52,9 @@ constexpr int WPE = FINESS_WPE;
 template <typename R, bool LXW>
 constexpr bool SEPARATE_FY = FINESS_STAGE_FY && !(LXW && sizeof(R) == sizeof(double));
 
-template <class P, typename R, int WK, bool LXW, int TI, int TJ>
+// LDSF: the Lax-Wendroff fluxes of the tile's stencils staged in LDS
+// (launch_lxw32), else read from memory at every stencil point.
+template <class P, typename R, int WK, bool LXW, int TI, int TJ, bool LDSF = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void k_stage2d(StageArgs a)
 {
     constexpr int NT = 256;
@@ -71,11 +73,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     constexpr bool SKIPPABLE = !(LXW && sizeof(R) == 4);
     R f3[3] = {R(0), R(0), R(0)};
     if constexpr (LXW && SKIPPABLE) lxw_fetch3<P, R, TI, TJ>(t, i0, j0, a, f3);
-    // the FP32 Lax-Wendroff form keeps its stencil fluxes in LDS (13 KB; four
-    // workgroups per CU remain)
-    constexpr bool FLUX_LDS = LXW && sizeof(R) == 4;
     const LxwTile<P, R, TI, TJ>* tile_flux = nullptr;
-    if constexpr (FLUX_LDS) {
+    if constexpr (LDSF) {
         __shared__ LxwTile<P, R, TI, TJ> lt;
         lxw_stage<P, R, TI, TJ>(t, i0, j0, a, lt);
         tile_flux = &lt;
@@ -160,13 +159,13 @@ static int launch_prim(const StageArgs& a, hipStream_t st)
     return launch_prim_tile<P, WK, LXW, 15, 16, true>(a, st);
 }
 
-template <class P, typename R, int WK, bool LXW, int TI, int TJ>
+template <class P, typename R, int WK, bool LXW, int TI, int TJ, bool LDSF = false>
 static int launch_stage(const StageArgs& a0, hipStream_t st)
 {
     StageArgs a = a0;
     const int nti = (a.mx + TI - 1) / TI, ntj = (a.my + TJ - 1) / TJ;
     a.ntj = ntj;
-    hipLaunchKernelGGL((k_stage2d<P, R, WK, LXW, TI, TJ>), dim3(nti * ntj), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((k_stage2d<P, R, WK, LXW, TI, TJ, LDSF>), dim3(nti * ntj), dim3(256), 0, st, a);
     return hipGetLastError() == hipSuccess ? 0 : -4;
 }
 
@@ -185,6 +184,23 @@ constexpr int STI = FINESS_STAGE_TI, STJ = FINESS_STAGE_TJ;
 #define FINESS_STAGE32_TJ 16
 #endif
 constexpr int STI32 = FINESS_STAGE32_TI, STJ32 = FINESS_STAGE32_TJ;
+
+// The FP32 Lax-Wendroff stage stages its stencil fluxes in LDS (13 KB more, 38
+// in all) from LXW32_LDS_CELLS cells on.  The states, the result and the fluxes
+// are 120 bytes a cell; while they fit the 256 MB of the Infinity Cache the
+// loads at every stencil point are served from L2 and it, and the smaller
+// workgroup hides them better.  Microseconds per stage, from memory and from
+// LDS: 400^2 20.9 / 23.6, 700^2 45.1 / 50.3, 1400^2 128 / 130, 1600^2
+// 169 / 172, 1700^2 203 / 197, 2048^2 295 / 275, 500 x 8000 281 / 264,
+// 4000 x 700 (2.8 million) 190 / 189.
+constexpr long long LXW32_LDS_CELLS = 2800000;
+
+static int launch_lxw32(const StageArgs& a, hipStream_t st)
+{
+    if ((long long)a.mx * a.my >= LXW32_LDS_CELLS)
+        return launch_stage<Euler2D, float, WENO_JS5_P2, true, STI32, STJ32, true>(a, st);
+    return launch_stage<Euler2D, float, WENO_JS5_P2, true, STI32, STJ32>(a, st);
+}
 
 template <class P, bool LXW>
 static int dispatch_prim(int wk, const StageArgs& a, hipStream_t st)
@@ -275,7 +291,7 @@ int launch_stage2d(int physics, int fp32, int wk, int lxw, const StageArgs& a, h
         if (!fp32 && lxw && a.face_x) return dispatch_limited(wk, a, st);
         if (!fp32) return lxw ? dispatch_prim<EulerPrim, true>(wk, a, st) : dispatch_prim<EulerPrim, false>(wk, a, st);
         if (wk != WENO_JS5_P2) return -1;
-        return lxw ? launch_stage<Euler2D, float, WENO_JS5_P2, true, STI32, STJ32>(a, st)
+        return lxw ? launch_lxw32(a, st)
                    : launch_stage<Euler2D, float, WENO_JS5_P2, false, STI32, STJ32>(a, st);
     }
     if (physics == PHYS_SHALLOW_WATER) {

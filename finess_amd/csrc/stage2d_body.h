@@ -588,6 +588,7 @@ __host__ __device__ __forceinline__ void phase_faces(int tid, int dir, int i0, i
     bool count = g.count;
     const WenoParams<R> wp{R(a.eps), R(a.power)};
     R fh[M];
+    const R amin = a.galpha ? R(a.galpha[dir]) : R(0);
     const R* lflux = static_cast<const R*>(dir ? a.lxw_G : a.lxw_F);
     if (tile) {
         using T = LxwTile<P, R, TI, TJ>;
@@ -597,7 +598,6 @@ __host__ __device__ __forceinline__ void phase_faces(int tid, int dir, int i0, i
         lstride = dir ? 1 : TJ;
     }
     // (skip3: a tile-uniform choice between two forms of the face code)
-    const R amin = a.galpha ? R(a.galpha[dir]) : R(0);
     const R alpha = skip3 ? face_flux<P, R, WK, LXW, S::NC, true>(sm.cv, base, stride, dir, lflux, lbase, lstride, lpl,
                                                                   a.pp, wp, R(a.alpha_scaling), fh, amin)
                           : face_flux<P, R, WK, LXW, S::NC>(sm.cv, base, stride, dir, lflux, lbase, lstride, lpl,
