@@ -35,10 +35,7 @@ struct BatchArgs {
 };
 
 // shapes the autotuner chooses from: (TI + 1) * TJ <= 256 and TI * (TJ + 1) <= 256
-// The first is the one a batch starts with: 15 x 16 has the fewest faces per
-// cell (2.13 against 2.17 of 7 x 32).  Microseconds per step, 15 x 16 against
-// 7 x 32: the shallow-water batch of 48 248 / 264 (FP32 stencils 255 / 276),
-// of 12 91 / 97, of 5 70 / 71.
+// (a batch starts with one of the first two: initial_shape)
 constexpr int BATCH_NSHAPES = 3;
 constexpr int BATCH_SHAPES[BATCH_NSHAPES][2] = {{15, 16}, {7, 32}, {3, 64}};
 
