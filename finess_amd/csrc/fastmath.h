@@ -72,6 +72,18 @@ __host__ __device__ __forceinline__ double sqrt_d(double x)
 #endif
 }
 
+// The binary exponent of x as frexp takes it (x 2^-exponent in [1/2, 1)).
+__host__ __device__ __forceinline__ int exponent(double x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_frexp_exp(x);
+#else
+    int e;
+    (void)frexp(x, &e);
+    return e;
+#endif
+}
+
 // An FP64 constant held in scalar registers.  Left as a literal it ties the
 // multiply-add to the two-operand form, which overwrites its addend: the
 // compiler then copies every addend that is used again (five copies for each
