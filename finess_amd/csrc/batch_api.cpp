@@ -190,6 +190,12 @@ int finess_batch_create(const finess_params* base, int nprob, const int* mx, con
         p.bc[1] == FINESS_BC_HOST || p.bc[2] == FINESS_BC_HOST || p.bc[3] == FINESS_BC_HOST ||
         (p.physics != FINESS_PHYS_SHALLOW_WATER && p.physics != FINESS_PHYS_EULER))
         return FINESS_ERR_CONFIG;
+    // periodic and reflecting ghosts are cells of the member within mbc of its
+    // side (bc_map): a smaller member has none, and the reads would leave its planes
+    for (int k = 0; k < nprob; k++)
+        if ((mx[k] >= 1 && mx[k] < p.mbc && (p.bc[0] != FINESS_BC_EXTRAP || p.bc[1] != FINESS_BC_EXTRAP)) ||
+            (my[k] >= 1 && my[k] < p.mbc && (p.bc[2] != FINESS_BC_EXTRAP || p.bc[3] != FINESS_BC_EXTRAP)))
+            return FINESS_ERR_CONFIG;
     if (finess_device_count() < 1) return FINESS_ERR_NODEVICE;
     finess_batch* b = new finess_batch();
     b->p = p;

@@ -329,7 +329,9 @@ int  finess_mlp_eval(finess_mlp* mlp, const float* X, long long n, int path, flo
  * tiles of all problems, each problem keeps its own a-posteriori CFL
  * controller on the device (accept/reject and dt from its own wave speeds),
  * and the step sequence is captured once in a HIP graph and replayed.  The
- * tile shape is chosen by finess_batch_autotune.  RK time stepping, 2D. */
+ * tile shape is chosen by finess_batch_autotune.  RK time stepping, 2D.  A
+ * member has at least mbc cells along a direction with a periodic or
+ * reflecting side (FINESS_ERR_CONFIG otherwise). */
 typedef struct finess_batch finess_batch;
 
 int  finess_batch_create(const finess_params* base, int nprob, const int* mx, const int* my, finess_batch** out);
