@@ -57,18 +57,6 @@ __host__ __device__ __forceinline__ void euler_flux(const T q[5], T gm1, T F[5],
     G[0] = ru2; G[1] = ru2 * u1; G[2] = ru2 * u2 + press; G[3] = ru2 * u3; G[4] = u2 * ep;
 }
 
-// Shallow water, g = 1 (apps/2d/shallow_water/lib/FluxFunc.cpp:8-35).
-template <typename T>
-__host__ __device__ __forceinline__ void sw_flux(const T q[3], T F[3], T G[3])
-{
-    const T h = q[0];
-    const T ih = hinv(h);
-    const T u1 = q[1] * ih, u2 = q[2] * ih;
-    const T hh = typename T::scalar(0.5) * (h * h);
-    F[0] = h * u1; F[1] = h * u1 * u1 + hh; F[2] = h * u1 * u2;
-    G[0] = h * u2; G[1] = h * u2 * u1; G[2] = h * u2 * u2 + hh;
-}
-
 // Hyper-dual number of scalar type T (double for the plain form, float for
 // the FP32 stencil form).
 template <typename T>
@@ -114,30 +102,6 @@ struct LxwPhys<Euler2D> {
         HDs<R> x[5];
         for (int m = 0; m < 5; m++) x[m] = HDs<R>(q[m], a[m], b[m], R(0));
         euler_flux<HDs<R>>(x, HDs<R>(R(pp.gamma - 1.0), R(0), R(0), R(0)), F, G);
-    }
-};
-
-// Shallow water: DFluxFunc / D2FluxFunc (apps/2d/shallow_water/lib/
-// DFluxFunc.cpp, D2FluxFunc.cpp) are the exact derivatives of the flux, so
-// the hyper-dual evaluation reproduces them.
-template <>
-struct LxwPhys<ShallowWater2D> {
-    static constexpr int M = 3;
-    template <typename R>
-    __host__ __device__ __forceinline__ static void flux(const R q[3], const PhysParams&, R F[3], R G[3])
-    {
-        const R h = q[0];
-        const R u1 = div_lp(q[1], h), u2 = div_lp(q[2], h);
-        F[0] = h * u1; F[1] = h * u1 * u1 + R(0.5) * h * h; F[2] = h * u1 * u2;
-        G[0] = h * u2; G[1] = h * u2 * u1; G[2] = h * u2 * u2 + R(0.5) * h * h;
-    }
-    template <typename R>
-    __host__ __device__ __forceinline__ static void flux_hd(const R q[3], const R a[3], const R b[3],
-                                                            const PhysParams&, HDs<R> F[3], HDs<R> G[3])
-    {
-        HDs<R> x[3];
-        for (int m = 0; m < 3; m++) x[m] = HDs<R>(q[m], a[m], b[m], R(0));
-        sw_flux<HDs<R>>(x, F, G);
     }
 };
 
@@ -233,7 +197,6 @@ template <class P, int TI, int TJ, typename R = double>
 __host__ __device__ __forceinline__ void lxw_phase_load(int tid, int e0i, int e0j, const LxwArgs& a,
                                                         LxwSmem<TI, TJ, P::MEQN, R>& sm)
 {
-    using S = LxwSmem<TI, TJ, P::MEQN, R>;
     LxwCells<P, TI, TJ> cells;
     cells.load(tid, e0i, e0j, a);
 #pragma unroll

@@ -170,8 +170,8 @@ static int pif_noc_stage_t(int wk, const PifArgs& a, hipStream_t st)
     switch (wk) {
     case WENO_JS5_P2: hipLaunchKernelGGL((k_pif_noc_faces<P, WENO_JS5_P2>), bf, blk, 0, st, a); break;
     case WENO_JS5_POW: hipLaunchKernelGGL((k_pif_noc_faces<P, WENO_JS5_POW>), bf, blk, 0, st, a); break;
-    case WENO_Z5: hipLaunchKernelGGL((k_pif_noc_faces<P, WENO_Z5>), bf, blk, 0, st, a); break;
-    case WENO_Z5_P2: hipLaunchKernelGGL((k_pif_noc_faces<P, WENO_Z5_P2>), bf, blk, 0, st, a); break;
+    case WENO_Z5:
+    case WENO_Z5_P2: hipLaunchKernelGGL((k_pif_noc_faces<P, WENO_Z5>), bf, blk, 0, st, a); break;
     case WENO_FD5: hipLaunchKernelGGL((k_pif_noc_faces<P, WENO_FD5>), bf, blk, 0, st, a); break;
     default: return -1;
     }

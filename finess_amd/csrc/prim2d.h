@@ -48,7 +48,6 @@ struct EulerPrim : Euler2D {
     static constexpr bool PRIM = true;
     static constexpr int NV = 6;  // rho, u, v, w, p, c
 
-    template <bool LP = false>
     __host__ __device__ __forceinline__ static void cell_record(const double q[5], const PhysParams& pp, double v[6])
     {
         const double ir = rcp_d(q[0]);
@@ -202,7 +201,6 @@ struct ShallowWaterPrim : ShallowWater2D {
     static constexpr bool PRIM = true;
     static constexpr int NV = 4;
 
-    template <bool LP = false>
     __host__ __device__ __forceinline__ static void cell_record(const double q[3], const PhysParams&, double v[4])
     {
         const double ih = rcp_d(q[0]);

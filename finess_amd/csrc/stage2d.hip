@@ -43,14 +43,11 @@ __device__ __forceinline__ void block_max2(A ax, A ay, unsigned long long* slot)
 #endif
 constexpr int WPE = FINESS_WPE;
 // The y-face fluxes in an LDS array of their own rather than in the x
-// fluxes' array after them (two barriers fewer, 10 KB more LDS in FP64, the
-// same 3 workgroups per CU): 1% less time for the FP32 Lax-Wendroff stage on
-// MI355X, but 3% more for the FP64 one, which keeps the shared array.
-#ifndef FINESS_STAGE_FY
-#define FINESS_STAGE_FY 1
-#endif
-template <typename R, bool LXW>
-constexpr bool SEPARATE_FY = FINESS_STAGE_FY && !(LXW && sizeof(R) == sizeof(double));
+// fluxes' array after them (two barriers fewer, 5 KB more LDS): 1% less time
+// for the FP32 Lax-Wendroff stage on MI355X, but 3% more for the FP64 one
+// (10 KB), which keeps the shared array.
+template <typename R>
+constexpr bool SEPARATE_FY = sizeof(R) == sizeof(float);
 
 // LDSF: the Lax-Wendroff fluxes of the tile's stencils staged in LDS
 // (launch_lxw32), else read from memory at every stencil point.
@@ -59,6 +56,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
 {
     constexpr int NT = 256;
     static_assert((TI + 1) * TJ <= NT && TI * (TJ + 1) <= NT, "one face per thread and direction");
+    static_assert(LXW || sizeof(R) == sizeof(float), "the FP64 Runge-Kutta stage is k_stage_prim");
     __shared__ StageSmem<P, R, TI, TJ> sm;
     if (stage_halted(a)) return;
     const int tile = xcd_remap(blockIdx.x, gridDim.x);
@@ -85,7 +83,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE))) void
     const bool skip3 = !__syncthreads_or(nz) && SKIPPABLE;
     R ax = R(0), ay = R(0);  // wave-speed maxima in the stencil precision
     double Lx[P::MEQN];
-    if constexpr (SEPARATE_FY<R, LXW>) {
+    if constexpr (SEPARATE_FY<R>) {
         // the y fluxes in an array of their own: both face passes run
         // without a barrier between them, and Lx is formed after them
         constexpr int NFY = TI * (TJ + 1);

@@ -108,7 +108,7 @@ __host__ __device__ __forceinline__ bool prim_load(int t, int i0, int j0, const 
         if (!ok[k]) continue;
         if constexpr (M == 5) nz3 = nz3 || q[k][3] != 0.0;
         double rec[P::NV];
-        P::template cell_record<>(q[k], a.pp, rec);
+        P::cell_record(q[k], a.pp, rec);
         for (int v = 0; v < P::NV; v++) cv[v][at[k]] = rec[v];
     }
     return nz3;
