@@ -98,6 +98,70 @@ void run_prim(const StageArgs& a, int two)
     else run_prim_tiles<P, WK, 7, 16, false>(a);
 }
 
+// The whole tile as prim_tile runs it, on the workgroup's real LDS layout
+// (PrimSmem, whose arrays overlay each other), one phase between two barriers
+// after the other.  The layout starts as NaN, so a read of what no phase has
+// written shows.
+template <class P, int WK, bool LXW, int PI, int PJ, bool TWO>
+void run_prim_overlay(const StageArgs& a)
+{
+    using S = PrimSmem<P, PI, PJ, TWO, LXW>;
+    constexpr int M = P::MEQN;
+    std::vector<S> smv(1);
+    S& sm = smv[0];
+    std::vector<double> fhv((size_t)PRIM_NT * M), ax(PRIM_NT), ay(PRIM_NT);
+    auto* fh = reinterpret_cast<double(*)[M]>(fhv.data());
+    for (int i0 = 0; i0 < a.mx; i0 += PI)
+        for (int j0 = 0; j0 < a.my; j0 += PJ) {
+            memset((void*)&sm, 0xff, sizeof sm);
+            bool nz = false;
+            const double *lF = nullptr, *lG = nullptr;
+            if constexpr (LXW) {
+                for (int t = 0; t < PRIM_NT; t++)
+                    nz = prim_load_fluxes<P, PI, PJ, S::NF, S::NG>(t, i0, j0, a, sm.x.F, sm.G) || nz;
+                lF = &sm.x.F[0][0];
+                lG = &sm.G[0][0];
+            }
+            for (int t = 0; t < PRIM_NT; t++) nz = prim_load<P, PI, PJ, S::NC>(t, i0, j0, a, sm.u.r.cv) || nz;
+            for (int t = 0; t < S::NT1; t++)
+                ax[t] = prim_face<P, WK, LXW, PI, PJ, 0, S::NC>(t, i0, j0, a, sm.u.r.cv, lF, !nz, fh[t]);
+            for (int t = 0; t < S::NFX; t++)
+                for (int m = 0; m < M; m++) sm.x.fx[m][t] = fh[t][m];
+            for (int t = 0; t < S::NT1; t++)
+                ay[t] = prim_face<P, WK, LXW, PI, PJ, 1, S::NC>(t, i0, j0, a, sm.u.r.cv, lG, !nz, fh[t]);
+            for (int t = 0; t < S::NFY; t++)
+                for (int m = 0; m < M; m++) sm.u.l.fy[m][t] = fh[t][m];
+            for (int t = 0; t < S::NT1; t++) {
+                sm.u.l.speed[0][t] = ax[t];
+                sm.u.l.speed[1][t] = ay[t];
+            }
+            for (int t = 0; t < S::NT1; t++) {
+                PrimUpdate<P, PI, PJ, 0, M> u;
+                u.load(t, i0, j0, a);
+                u.store(a, stage_bdt(a), sm.x.fx, sm.u.l.fy);
+            }
+        }
+}
+
+template <class P, bool LXW, int PI, int PJ, bool TWO>
+void dispatch_overlay(int wk, const StageArgs& a)
+{
+    switch (wk) {
+    case WENO_FD5: run_prim_overlay<P, WENO_FD5, LXW, PI, PJ, TWO>(a); break;
+    case WENO_Z5: run_prim_overlay<P, WENO_Z5, LXW, PI, PJ, TWO>(a); break;
+    case WENO_Z5_P2: run_prim_overlay<P, WENO_Z5_P2, LXW, PI, PJ, TWO>(a); break;
+    case WENO_JS5_POW: run_prim_overlay<P, WENO_JS5_POW, LXW, PI, PJ, TWO>(a); break;
+    default: run_prim_overlay<P, WENO_JS5_P2, LXW, PI, PJ, TWO>(a); break;
+    }
+}
+
+template <class P, bool LXW>
+void dispatch_overlay(int wk, const StageArgs& a, int two)
+{
+    if (two) dispatch_overlay<P, LXW, 15, 16, true>(wk, a);
+    else dispatch_overlay<P, LXW, 7, 16, false>(wk, a);
+}
+
 template <class P>
 void dispatch_prim(int wk, const StageArgs& a, int two)
 {
@@ -250,6 +314,27 @@ int emu_construct_integrated_r(const finess_params* p, double dt, const double* 
                 F[((i + g) * ldq + (j + g)) * M + m] = Fo[o];
                 G[((i + g) * ldq + (j + g)) * M + m] = Go[o];
             }
+    return 0;
+}
+
+// The same on the tile's real LDS layout; F, G (extended-grid planes): the
+// Lax-Wendroff form, null: Runge-Kutta.
+int emu_prim_overlay(const finess_params* p, const double* q, const double* F, const double* G, int two, double* L)
+{
+    StageArgs a;
+    memset(&a, 0, sizeof a);
+    a.src = q; a.mx = p->mx; a.my = p->my; a.plane = (long long)p->mx * p->my;
+    for (int k = 0; k < 4; k++) a.bc[k] = p->bc[k];
+    a.dx = p->dx; a.dy = p->dy; a.idx = 1.0 / p->dx; a.idy = 1.0 / p->dy;
+    a.alpha_scaling = p->alpha_scaling; a.eps = p->epsilon; a.power = p->power_param;
+    a.pp.gamma = p->gamma; a.pp.sw_compat_hl = p->sw_compat_hl;
+    a.Lout = L; a.lxw_F = F; a.lxw_G = G;
+    int wk = wk_of(p);
+    if (wk == WENO_Z5) wk = weno_z5_kind(p->power_param, p->epsilon);
+    if (p->physics == FINESS_PHYS_EULER && F) dispatch_overlay<EulerPrim, true>(wk, a, two);
+    else if (p->physics == FINESS_PHYS_EULER) dispatch_overlay<EulerPrim, false>(wk, a, two);
+    else if (F) dispatch_overlay<ShallowWaterPrim, true>(wk, a, two);
+    else dispatch_overlay<ShallowWaterPrim, false>(wk, a, two);
     return 0;
 }
 
