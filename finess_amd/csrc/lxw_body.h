@@ -8,8 +8,10 @@
 //
 // with A_d the flux Jacobians and H_d(a, b) their second derivatives applied
 // to two vectors.  The reference forms A and H as explicit tensors from the
-// app's DFluxFunc / D2FluxFunc and contracts them; here every product is a
-// directional derivative of the flux itself, evaluated exactly with
+// app's DFluxFunc / D2FluxFunc and contracts them.  The FP64 form of the
+// unlimited step writes the products out (lxw64_cell); in the FP32 form and the
+// limited step every product is a directional derivative of the flux itself,
+// evaluated exactly with
 // hyper-dual numbers (x + a e1 + b e2 + ab e1e2, e1^2 = e2^2 = 0): one flux
 // evaluation at q + a e1 + b e2 yields A a (e1 part), A b (e2 part) and
 // H(a, b) (e1e2 part).  Derivatives: 5-point central differences Diff1/Diff2

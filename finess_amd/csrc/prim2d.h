@@ -1,7 +1,7 @@
 // prim2d.h -- the fused FP64 face: characteristic WENO5-LLF on primitive cell
 // records (lib/2d/ConstructL.cpp:63-208 for x, :215-358 for y), for 2D Euler
 // and shallow water.  Used by the plain and batched FP64 stages and, with
-// fluxes read from memory, by the Lax-Wendroff and RK4-PIF stages.
+// given fluxes, by the Lax-Wendroff and RK4-PIF stages.
 //
 // The stage is bound by FP64 instruction issue, so the face is arranged for
 // the fewest instructions and LDS reads.  With (u1, u2, u3) the mean velocity
@@ -21,7 +21,7 @@
 // other in a rolled loop (unrolled, both parts' values are live and the kernel
 // takes 194 registers instead of 128).
 //
-// Euler, Runge-Kutta, 1024^2: 25.8 M VALU instructions and 59 us per stage
+// Euler, Runge-Kutta, 1024^2: 25.6 M VALU instructions and 59 us per stage
 // (40.6 M and 88 us with conserved records and the reconstruction of weno5);
 // shallow water 43 us (71; its flux divided by h at every stencil cell).
 #pragma once
@@ -58,8 +58,9 @@ struct EulerPrim : Euler2D {
     }
 
     // Flux of one face; cv: records, the stencil cell s at base + s * stride
-    // (cells i-3..i+2).  LXW: the stencil fluxes come from memory (flux of
-    // cell s and field k at lflux[k * lplane + lbase + s * lstride]).
+    // (cells i-3..i+2).  LXW: the stencil fluxes are given (flux of cell s
+    // and field k at lflux[k * lplane + lbase + s * lstride]; the tile keeps
+    // them in LDS).
     // SKIP3: every stencil cell (and flux) has zero rho w.  Returns alpha.
     template <int WK, bool LXW, bool SKIP3, int NC>
     __device__ __host__ __forceinline__ static double face(const double (*cv)[NC], int base, int stride, int dir,

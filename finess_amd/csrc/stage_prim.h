@@ -271,7 +271,7 @@ __device__ __forceinline__ void prim_tile(int t, int i0, int j0, const StageArgs
     bool nz = false;
     // beta dt is read before the tile's cells, not where the update needs it: the
     // registers then fit without spills (450^2 61.2 -> 58.8 us per step, 128^2
-    // 22.1 -> 21.7, 2048^2 652 -> 645; the ninth order the same)
+    // 22.1 -> 21.7, 2048^2 652 -> 645)
     const double bdt = stage_bdt(a);
     const double *lF = nullptr, *lG = nullptr;
     if constexpr (LXW) {

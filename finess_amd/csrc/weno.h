@@ -154,8 +154,8 @@ __host__ __device__ __forceinline__ R weno5(const R g[5], const WenoParams<R>& w
 //     beta_0 = 4/3 (d0^2 - 11/4 d0 d1 + 5/2 d1^2),
 //     beta_1 = 4/3 (d1^2 -  5/4 d1 d2 +     d2^2),
 //     beta_2 = 4/3 (d3^2 - 11/4 d3 d2 + 5/2 d2^2),
-// (smallest eigenvalue 0.18 of the largest coefficient: no digit is lost that
-// the sum of squares keeps), and the candidates are g[2] plus two of them.
+// (the outer forms' eigenvalues are 0.18 and 3.3, so their cancellation costs at
+// most a factor of 18), and the candidates are g[2] plus two of them.
 // The common factor 4/3 leaves every weight ratio unchanged, so it is dropped
 // and eps is scaled by 3/4 instead.  The reconstruction of a fused stage takes
 // 36 FP64 instructions and one reciprocal estimate, where the form above takes
@@ -181,7 +181,7 @@ __host__ __device__ __forceinline__ double weno5_fp64(const double g[5], double 
     const double a0 = fma(d0, fma(c1, d1, d0), fma(c3, p1, e));
     const double a1 = fma(d1, fma(c2, d2, d1), fma(d2, d2, e));
     const double a2 = fma(d3, fma(c1, d2, d3), fma(c3, p2, e));
-    // candidate minus g[2], times the linear weight's share (0.1, 0.6, 0.3 -> 1, 1/6 .. folded below)
+    // candidate minus g[2], times its linear weight over 0.1 (1, 6 and 3)
     const double v0 = fma(5.0 / 6.0, d1, (-1.0 / 3.0) * d0);
     const double v1 = fma(2.0, d2, d1);
     const double v2 = fma(2.0, d2, -0.5 * d3);
