@@ -1849,23 +1849,30 @@ static int advance_dev(finess_ctx* c, double tend, double* dtv, long long fixed_
     return rc;
 }
 
-// Whether the steps' controller runs on the device: the schemes whose kernels
-// all take dt and the halt word from the control block.  (SSP(10,4) in 1D and
-// with routing, the fifth-order scheme, RK4-PIF and the limited step keep the
-// host's, which waits for the device after each step.)  Microseconds per step
-// with the host's controller and the device's: Lax-Wendroff 100^2 27.5 / 17.3,
-// 400^2 44.2 / 34.0; SSP(10,4) 333 x 217 123 / 113.
-static bool device_controlled(const finess_params& p)
+// Whether the controller of a run that takes about `steps` steps at its first
+// dt runs on the device: the schemes whose kernels all take dt and the halt
+// word from the control block.  (SSP(10,4) in 1D and with routing, the
+// fifth-order scheme, RK4-PIF and the limited step keep the host's, which waits
+// for the device after each step.)  The control block's upload and its read-back
+// cost more than the waits of a few steps: SSP(10,4) and Lax-Wendroff keep the
+// host's below SHORT_RUN steps.  Microseconds per call with the host's and the
+// device's, 1, 4 and 8 steps: Lax-Wendroff 128^2 30 / 43, 112 / 117, 221 / 190,
+// 600^2 69 / 82, 262 / 263, 511 / 475; SSP(10,4) 128^2 83 / 115, 314 / 313,
+// 617 / 586.
+static bool device_controlled(const finess_params& p, double steps)
 {
+    constexpr double SHORT_RUN = 6.0;
     if (p.verbosity || p.host_controller) return false;
-    if (p.time_stepping_method == FINESS_TS_LXW) return p.ndims == 2 && !p.mpp_limiter;
+    if (p.time_stepping_method == FINESS_TS_LXW) return p.ndims == 2 && !p.mpp_limiter && steps >= SHORT_RUN;
     if (p.time_stepping_method != FINESS_TS_RK) return false;
-    return p.time_order <= 3 || (p.time_order == 4 && p.ndims == 2 && p.routing == FINESS_ROUTE_NONE);
+    return p.time_order <= 3 ||
+           (p.time_order == 4 && p.ndims == 2 && p.routing == FINESS_ROUTE_NONE && steps >= SHORT_RUN);
 }
 
 static int advance_impl(finess_ctx* c, double tend, double* dtv, long long fixed_steps, finess_stats* stats)
 {
-    if (c && dtv && c->have_state && c->ctl && device_controlled(c->p) && !c->hostbc)
+    if (c && dtv && c->have_state && c->ctl && !c->hostbc &&
+        device_controlled(c->p, fixed_steps > 0 ? (double)fixed_steps : (tend - c->t) / dtv[1]))
         return advance_dev(c, tend, dtv, fixed_steps, stats);
     if (!c || !dtv) return FINESS_ERR_ARG;
     if (!c->have_state) return fail(c, FINESS_ERR_ARG, "no state");
