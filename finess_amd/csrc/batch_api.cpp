@@ -115,10 +115,11 @@ int set_shape(finess_batch* b, int shape)
     return upload_table(b);
 }
 
-// The shape that a batch starts with: 15 x 16 where it gives the fullest CU
-// fewer workgroups than 7 x 32 (a tile of either takes about as long), or, with
-// no more than one workgroup a CU, where it has fewer tiles.  Microseconds per
-// stage, 15 x 16 / 7 x 32, with their tiles:
+// The shape that a batch starts with: 15 x 16 where it has fewer tiles than
+// 7 x 32 (a tile of either takes about as long).  With all tiles resident at
+// once the launch lasts as long as the fullest CU: there 15 x 16 has to give
+// that one fewer workgroups, or every CU at most one.  Microseconds per stage,
+// 15 x 16 / 7 x 32, with their tiles:
 //   FP64 shallow water  48 members of 64 to 390 cells a side (10255, 11367) 113 / 121,
 //                       12 smaller ones (1415, 1551) 19 / 24, 900 x 7 (8 x 60, 8 x 129) 10 / 16,
 //                       100 of 32^2 (600, 500) 11 / 9, 100 of 7 x 900 (5700, 2900) 47 / 38
@@ -128,15 +129,18 @@ int initial_shape(const finess_batch* b)
 {
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device) != hipSuccess || cus < 1) return 0;
-    long long tiles[2];
+    long long tiles[2], most[2];
+    bool resident = true;
     for (int s = 0; s < 2; s++) {
         tiles[s] = 0;
         for (const BatchProb& pr : b->host)
             tiles[s] += (long long)((pr.mx + BATCH_SHAPES[s][0] - 1) / BATCH_SHAPES[s][0]) *
                         ((pr.my + BATCH_SHAPES[s][1] - 1) / BATCH_SHAPES[s][1]);
+        most[s] = (tiles[s] + cus - 1) / cus;
+        resident = resident && tiles[s] <= batch_grid(b->physics, b->fp32, s, b->device);
     }
-    const long long most0 = (tiles[0] + cus - 1) / cus, most1 = (tiles[1] + cus - 1) / cus;
-    return most0 < most1 || (most0 == 1 && most1 == 1 && tiles[0] < tiles[1]) ? 0 : 1;
+    if (tiles[0] >= tiles[1]) return 1;
+    return resident && most[0] == most[1] && most[0] > 1 ? 1 : 0;
 }
 
 int enqueue_steps(finess_batch* b, int steps)
